@@ -1639,7 +1639,8 @@ int dp_wa_forward_tiles(int dtype, int model, const void* pos, int64_t num_nodes
   DP_PROBE_OP(DP_OP_WA_FORWARD, s);
   double* partials = (double*)workspace;
   char* pin_xy = (char*)workspace + reduce_slot_bytes();
-  const int g1 = (int)num_net_tiles;
+  // as many partial sums as dp_wa_num_partials says: without a net tile one of 0
+  const int g1 = num_net_tiles > 0 ? (int)num_net_tiles : 1;
   const int g2 = num_big > 0 ? grid_cap(num_big, 4, kBigGrid) : 0;
   return DP_DISPATCH(dtype, name, [&] {
     typedef typename Vec2<T>::type V;
@@ -1672,7 +1673,10 @@ int dp_wa_forward_tiles(int dtype, int model, const void* pos, int64_t num_nodes
     auto bignet = model == DP_WL_LOGSUMEXP                 ? k_wa_big<T, kWaLse, int>
                   : model == DP_WL_WEIGHTED_AVERAGE_CENTRED ? k_wa_big<T, kWaCentred, int>
                                                             : k_wa_big<T, kWaRef, int>;
-    if (g1 > 0) {
+    if (num_net_tiles == 0) {
+      hipLaunchKernelGGL(k_fill<double>, dim3(1), dim3(64), 0, s, partials, (int64_t)1, 0.0);
+      DP_LAUNCHED("partial sum of no net tile");
+    } else {
       DP_PROBED(DP_KERNEL_WA_FORWARD, s,
                 hipLaunchKernelGGL(tiled, dim3(g1), dim3(TileBlock<T>::value), 0, s, a,
                                    (const int2*)net_tiles, net_cell, Runs{net_chunk, net_delta},
