@@ -165,7 +165,9 @@ static TiledLayout tiled_layout(int nbx, int nby, int64_t ncells, size_t tsize, 
   L.ntx = (int)ceil_div(nbx, kTile);
   L.nty = (int)ceil_div(nby, kTile);
   L.ntiles = L.ntx * L.nty;
-  L.max_work = ceil_div(ncells, chunk_cells(ncells)) + 2 * (int64_t)L.ntiles + 1;
+  // room for items of the smaller size at every count, so that the workspace never
+  // shrinks as the count grows (a caller may size it by more nodes than it bins)
+  L.max_work = ceil_div(ncells, kChunk / 2) + 2 * (int64_t)L.ntiles + 1;
   const size_t n = (size_t)(ncells > 0 ? ncells : 1);
   size_t o = 0;
   L.off_count = o;  // cells per (class, tile)
