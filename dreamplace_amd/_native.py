@@ -235,10 +235,11 @@ def as_i32(t):
 
 
 def as_u8(t):
-    """A mask as bytes of 0 and 1: a bool tensor's own storage, else a copy."""
+    """A mask as bytes of 0 and 1, a bool tensor's in a copy: what becomes of it
+    between a forward and its backward stays out of the latter."""
     if t is None or t.dtype == torch.uint8:
         return t
-    return t.view(torch.uint8) if t.dtype == torch.bool else t.to(torch.uint8)
+    return t.to(torch.uint8)
 
 
 class Derived:

@@ -35,7 +35,7 @@ class HPWL(nn.Module):
         self.netpin_start = N.as_i32(netpin_start)
         self.pin2net_map = pin2net_map
         self.net_weights = net_weights
-        self.net_mask = net_mask.to(torch.uint8)
+        self.net_mask = N.as_u8(net_mask)
         self.algorithm = algorithm
 
     def forward_fp64(self, pos):
