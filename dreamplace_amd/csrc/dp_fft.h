@@ -76,6 +76,16 @@ int fft_poisson(const void* plan, int M, int N, const void* map, double bsx, dou
                 bool want_phi, void* field_x, void* field_y, void* potential, void* energy,
                 void* ws, size_t slab, hipStream_t s);
 
+// An energy term c K a^2, from the type's a and k: in FP64, K by a Newton step from
+// k (2^-22 -> 2^-44), as the terms of few modes are most of the sum and the FP32
+// step du alone shifts each by 1e-7.
+template <typename T>
+__device__ __forceinline__ double energy_term(T c, T k, double wu, double wv, T a) {
+  double kd = (double)k;
+  if constexpr (sizeof(T) == 4) kd = fma(kd, fma(-fma(wu, wu, wv * wv), kd, 1.0), kd);
+  return (double)c * kd * ((double)a * (double)a);
+}
+
 #ifdef DP_FFT_IMPL
 
 template <typename T>
@@ -546,7 +556,8 @@ __device__ __forceinline__ T spectral_k(T wu, T wv) {
 template <typename T, int LG, int F>
 __global__ void __launch_bounds__(2 * F * Fft<LG>::threads)
     k_fft_cols_solve(const T* __restrict__ A, typename Vec2<T>::type* field, T* phi, int N,
-                     T scale, double mean_scale, const double* __restrict__ row_mean, T du, T dv,
+                     T scale, double mean_scale, const double* __restrict__ row_mean, double du,
+                     double dv,
                      double* partials, const typename Vec2<T>::type* __restrict__ tw,
                      const typename Vec2<T>::type* __restrict__ dw) {
   typedef typename Vec2<T>::type V;
@@ -599,7 +610,7 @@ __global__ void __launch_bounds__(2 * F * Fft<LG>::threads)
   const int c = t % F, cj = t / F;  // cj < 2P
   Cx<T> z[2][4];                    // [pair][column, k | n - k]
   Cx<T> zp[2][2];                   // the potential's
-  T esum = 0;
+  double esum = 0;
 #pragma unroll
   for (int m = 0; m < 2; ++m) {
     const int k = cj + 2 * m * P, nk = k ? n - k : n / 2;
@@ -607,16 +618,16 @@ __global__ void __launch_bounds__(2 * F * Fft<LG>::threads)
     const Cx<T> w = ld2<T>(dw + k);
     DctPair<T> d = dct_pair<T>(ld2<T>(b + fpad(k)), ld2<T>(b + fpad(nk)), w, k);
     const int v = g0 + 2 * c;
-    const T wk = du * (T)k, wnk = du * (T)nk;
+    const T wk = (T)du * (T)k, wnk = (T)du * (T)nk;
     DctPair<T> ph;
 #pragma unroll
     for (int col = 0; col < 2; ++col) {
-      const T wv = dv * (T)(v + col);
+      const T wv = (T)dv * (T)(v + col);
       const T ak = (col ? d.bk : d.ak) * scale, ank = (col ? d.bnk : d.ank) * scale;
       const T kk = spectral_k(wk, wv), knk = spectral_k(wnk, wv);
       const T cv = v + col ? T(2) : T(1), ck = k ? T(2) : T(1);
-      esum += (ck * cv * kk) * ak * ak;
-      esum += (T(2) * cv * knk) * ank * ank;
+      esum += energy_term<T>(ck * cv, kk, du * k, dv * (v + col), ak);
+      esum += energy_term<T>(T(2) * cv, knk, du * nk, dv * (v + col), ank);
       DctPair<T> q;
       q.ak = ak * (wk * kk * (T)0.5);  // field x, IDXST: k and n - k swapped
       q.ank = ank * (wnk * knk * (T)0.5);
@@ -687,7 +698,7 @@ __global__ void __launch_bounds__(2 * F * Fft<LG>::threads)
     }
   }
   if (partials) {
-    const double s = wave_sum((double)esum);
+    const double s = wave_sum(esum);
     __syncthreads();
     if ((t & 63) == 0) red[t >> 6] = s;
     __syncthreads();
@@ -858,8 +869,8 @@ int fft_poisson(const void* plan, int M, int N, const void* map, double bsx, dou
       blocks = N / (2 * F);
       hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(2 * F * Fft<LG>::threads), lds, s,
                          (const T*)A, field, ph, N, (T)(2.0 / M), 2.0 * inv_area,
-                         (const double*)row_mean, (T)(2.0 * M_PI / M),
-                         (T)(2.0 * M_PI / N * (bsx / bsy)), part, tb.tw_m, tb.dw_m);
+                         (const double*)row_mean, 2.0 * M_PI / M, 2.0 * M_PI / N * (bsx / bsy), part,
+                         tb.tw_m, tb.dw_m);
       DP_LAUNCHED("k_fft_cols_solve");
       return DP_OK;
     };

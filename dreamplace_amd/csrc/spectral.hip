@@ -969,7 +969,6 @@ __global__ void __launch_bounds__(256) k_gemm_any(GemmBatch bt, GemmExtra ex) {
   __syncthreads();
   // wavefront w finishes accumulator elements w, w + 4, ... of every lane
   double e = 0;
-  T es = 0;
 #pragma unroll
   for (int x = 0; x < WT * WT; ++x) {
     const int t = x * 4 + w, i = x / WT, j = x % WT;
@@ -983,13 +982,13 @@ __global__ void __launch_bounds__(256) k_gemm_any(GemmBatch bt, GemmExtra ex) {
       ((T*)ex.ax)[o] = v * m.kx;
       ((T*)ex.ay)[o] = v * m.ky;
       if (ex.ak) ((T*)ex.ak)[o] = v * m.k;
-      es += m.e * v * v;
+      e += energy_term<T>((row ? T(2) : T(1)) * (col ? T(2) : T(1)), m.k, ex.du * row, ex.dv * col, v);
     } else {
       ((T*)gd.C)[o] = v;
       if (gd.R) e += (double)v * (double)((const T*)gd.R)[o];
     }
   }
-  if (kWeights) e = (double)es * ((double)M * N / 4.0);
+  if (kWeights) e *= (double)M * N / 4.0;
   if (gd.partials) {
     const double bs = block_sum<256>(e, smem);
     if (threadIdx.x == 0) gd.partials[tile] = bs;
