@@ -243,24 +243,26 @@ def as_u8(t):
 
 
 class Derived:
-    """A tensor computed once from static index maps and kept while they are
+    """Tensors computed once from static index maps and kept while they are
     the same objects, unmodified: get(build, *maps).  It holds the maps, so
     none can be replaced by another at its address, and rebuilds after an
     in-place change.  A build is waited for, so that any stream may use it.
-    Of inference tensors, whose changes are not counted, nothing is kept."""
+    get is None where nothing may be kept, and the caller works on the maps
+    themselves: of inference tensors, whose changes are not counted, and while
+    a graph is captured, which would only record a build and would hold the
+    addresses of what a later change of the maps frees."""
 
     def __init__(self):
         self._state = (None, None, None)  # maps, their versions, the value
 
     def get(self, build, *maps):
-        if any(m.is_inference() for m in maps):
-            return build(*maps)
+        if any(m.is_inference() for m in maps) or torch.cuda.is_current_stream_capturing():
+            return None
         versions = tuple(m._version for m in maps)
         held, seen, value = self._state
         if held is None or any(a is not b for a, b in zip(held, maps)) or seen != versions:
             value = build(*maps)
-            if not torch.cuda.is_current_stream_capturing():
-                torch.cuda.current_stream(maps[0].device).synchronize()
+            torch.cuda.current_stream(maps[0].device).synchronize()
             self._state = (maps, versions, value)
         return value
 

@@ -93,17 +93,15 @@ class PinPos(nn.Module):
 
     def _plan(self, dtype):
         """exchange.pin_tiles of the maps, or None where the plain kernels are
-        taken: few pins, maps that the tiles do not apply to, or inference
-        tensors, of which no plan is kept."""
+        taken: few pins, maps that the tiles do not apply to, or where no plan
+        is kept (_native.Derived)."""
         maps = self.pin2node_map, self.flat_node2pin_map, self.flat_node2pin_start_map
-        if (maps[0].numel() < TILE_MIN_PINS or not all(m.is_cuda for m in maps)
-                or any(m.is_inference() for m in maps)):
+        if maps[0].numel() < TILE_MIN_PINS or not all(m.is_cuda for m in maps):
             return None
         cap = N.query("dp_wa_tile_pins", N.DP_FLOAT64 if dtype == torch.float64 else N.DP_FLOAT32)
         sizes = cap, int(self.num_physical_nodes)
-        of, plan = self._tiles.get(lambda *m: (sizes, exchange.pin_tiles(cap, *m, sizes[1])),
-                                   *maps)
-        return plan if of == sizes else None
+        kept = self._tiles.get(lambda *m: (sizes, exchange.pin_tiles(cap, *m, sizes[1])), *maps)
+        return kept[1] if kept is not None and kept[0] == sizes else None
 
     def forward(self, pos):
         assert pos.numel() % 2 == 0

@@ -30,7 +30,8 @@ class PinWeightSum(nn.Module):
     def _nets(self):
         """(the net of every node-order pin slot - the two maps in one - or
         None, exchange.weight_tiles of it or None), laid out once, one of the
-        two; None for maps off the GPU."""
+        two; neither where nothing is kept of the maps (_native.Derived); None
+        for maps off the GPU."""
         maps = self.flat_nodepin, self.pin2net_map, self.nodepin_start
         if not all(m.is_cuda for m in maps):
             return None
@@ -38,11 +39,11 @@ class PinWeightSum(nn.Module):
         def build(pins, nets, start):
             slot_net = nets[pins.long()].contiguous()
             x = None
-            if pins.numel() >= TILE_MIN_PINS and not any(m.is_inference() for m in maps):
+            if pins.numel() >= TILE_MIN_PINS:
                 x = exchange.weight_tiles(N.query("dp_wa_tile_pins", N.DP_FLOAT32), slot_net, start)
             return (slot_net, None) if x is None else (None, x)
 
-        return self._plan.get(build, *maps)
+        return self._plan.get(build, *maps) or (None, None)
 
     def forward(self, net_weights):
         N.require_gpu(net_weights, name="PinWeightSum")
@@ -61,7 +62,10 @@ class PinWeightSum(nn.Module):
                    N.ptr(x["cell"]), N.ptr(x["chunk"]), N.ptr(x["delta"]), N.ptr(x["node_tiles"]),
                    len(x["node_tiles"]) - 1, N.ptr(x["node_cell"]), N.ptr(self.nodepin_start),
                    nphys, n, N.ptr(ws), N.ptr(out), s)
-        else:
+        elif nets is not None:
             N.call("dp_pin_weight_sum_slots", code, N.ptr(w), N.ptr(nets),
                    N.ptr(self.nodepin_start), nphys, n, N.ptr(out), s)
+        else:
+            N.call("dp_pin_weight_sum", code, N.ptr(w), N.ptr(self.flat_nodepin),
+                   N.ptr(self.nodepin_start), N.ptr(self.pin2net_map), nphys, n, N.ptr(out), s)
         return out
