@@ -30,13 +30,16 @@ class PinWeightSum(nn.Module):
     def _nets(self):
         """(the net of every node-order pin slot - the two maps in one - or
         None, exchange.weight_tiles of it or None), laid out once, one of the
-        two; neither where nothing is kept of the maps (_native.Derived); None
-        for maps off the GPU."""
+        two; neither where nothing is kept of the maps (_native.Derived) or
+        they hold more than pins; None for maps off the GPU."""
         maps = self.flat_nodepin, self.pin2net_map, self.nodepin_start
         if not all(m.is_cuda for m in maps):
             return None
 
         def build(pins, nets, start):
+            # what lies past the nodes' lists is never read and may name no pin
+            if not bool(((pins >= 0) & (pins < nets.numel())).all()):
+                return None, None
             slot_net = nets[pins.long()].contiguous()
             x = None
             if pins.numel() >= TILE_MIN_PINS:

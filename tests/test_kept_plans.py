@@ -101,3 +101,18 @@ def test_capture(gpu, monkeypatch, least):
         check(out, sums)
         other_maps()
         check(a(pos), b(w))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("least", [1, 1 << 40], ids=["tiles", "few"])
+@pytest.mark.parametrize("past", [-1, 1 << 30])
+def test_padded_map(gpu, monkeypatch, past, least):
+    """A node-to-pin map longer than its start array says, the rest no pin."""
+    from dreamplace_amd import pin_weight_sum
+    print("case padded map %d %d" % (past, least), flush=True)
+    monkeypatch.setattr(pin_weight_sum, "TILE_MIN_PINS", least)
+    p2n, order, start, p2e = netlist(gpu, 5000, 700, 900)
+    w = torch.rand(900, device=gpu)
+    want = pin_weight_sum.PinWeightSum(order, start, p2e, 800)(w)
+    padded = torch.cat([order, order.new_full((100,), past)])
+    assert torch.equal(pin_weight_sum.PinWeightSum(padded, start, p2e, 800)(w), want)
