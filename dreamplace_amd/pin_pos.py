@@ -105,6 +105,9 @@ class PinPos(nn.Module):
 
     def forward(self, pos):
         assert pos.numel() % 2 == 0
+        # the node tiles hold every physical node, with or without pins
+        whole = pos.numel() >= 2 * int(self.num_physical_nodes)
         return PinPosFunction.apply(pos, self.pin_offset_x, self.pin_offset_y, self.pin2node_map,
                                     self.flat_node2pin_map, self.flat_node2pin_start_map,
-                                    self.num_physical_nodes, self._plan(pos.dtype))
+                                    self.num_physical_nodes,
+                                    self._plan(pos.dtype) if whole else None)

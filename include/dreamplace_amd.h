@@ -345,7 +345,8 @@ int dp_pin_pos_backward(int dtype, const void* grad_pin_pos, int64_t num_pins,
  * place_node, its runs); the other order's tile t is the pins_per_tile pins
  * from t * pins_per_tile on, so a pin's position has its place among the same
  * numbers: pin_cell[position's place] = pin - its tile's first, with the runs of
- * derivative's places (pin_chunk, pin_delta).  workspace:
+ * derivative's places (pin_chunk, pin_delta).  The tiles' nodes, with or without
+ * pins, are read: num_nodes is no less than theirs.  workspace:
  * dp_pin_pos_workspace_bytes(dtype, num_pins). */
 size_t dp_pin_pos_workspace_bytes(int dtype, int64_t count);
 int dp_pin_pos_forward_tiles(int dtype, const void* pos, int64_t num_nodes,

@@ -116,3 +116,18 @@ def test_padded_map(gpu, monkeypatch, past, least):
     want = pin_weight_sum.PinWeightSum(order, start, p2e, 800)(w)
     padded = torch.cat([order, order.new_full((100,), past)])
     assert torch.equal(pin_weight_sum.PinWeightSum(padded, start, p2e, 800)(w), want)
+
+
+def test_few_positions(monkeypatch):
+    """Positions of fewer nodes than the physical ones, the last of which have no
+    pins: no node tile, which reads all of them."""
+    from dreamplace_amd import pin_pos
+    p2n = torch.arange(12) % 3
+    start = torch.tensor([0, 4, 8, 12, 12, 12])
+    op = pin_pos.PinPos(torch.rand(12), torch.rand(12), p2n, p2n.argsort(stable=True), start, 5)
+    monkeypatch.setattr(op, "_plan", lambda dtype: "tiles")
+    taken = []
+    monkeypatch.setattr(pin_pos.PinPosFunction, "apply", lambda *a: taken.append(a[-1]))
+    for nodes in (3, 4, 5, 6):
+        op(torch.rand(2 * nodes))
+    assert taken == [None, None, "tiles", "tiles"]
