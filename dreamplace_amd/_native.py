@@ -244,26 +244,31 @@ def as_u8(t):
 
 class Derived:
     """Tensors computed once from static index maps and kept while they are
-    the same objects, unmodified: get(build, *maps).  It holds the maps, so
-    none can be replaced by another at its address, and rebuilds after an
-    in-place change.  A build is waited for, so that any stream may use it.
+    the same objects, unmodified and at the same addresses: get(build, *maps).
+    It holds the maps, so none can be replaced by another, and rebuilds after
+    an in-place change (one that torch does not count, through .data or a raw
+    pointer, is not seen).  A build is waited for, so that any stream may use
+    it.  A copy or a saved one holds nothing.
     get is None where nothing may be kept, and the caller works on the maps
     themselves: of inference tensors, whose changes are not counted, and while
     a graph is captured, which would only record a build and would hold the
     addresses of what a later change of the maps frees."""
 
     def __init__(self):
-        self._state = (None, None, None)  # maps, their versions, the value
+        self._state = (None, None, None)  # maps, their versions and addresses, the value
+
+    def __reduce__(self):
+        return Derived, ()  # a copied map's versions start anew
 
     def get(self, build, *maps):
         if any(m.is_inference() for m in maps) or torch.cuda.is_current_stream_capturing():
             return None
-        versions = tuple(m._version for m in maps)
+        key = tuple((m._version, m.data_ptr()) for m in maps)
         held, seen, value = self._state
-        if held is None or any(a is not b for a, b in zip(held, maps)) or seen != versions:
+        if held is None or any(a is not b for a, b in zip(held, maps)) or seen != key:
             value = build(*maps)
             torch.cuda.current_stream(maps[0].device).synchronize()
-            self._state = (maps, versions, value)
+            self._state = (maps, key, value)
         return value
 
 

@@ -1,5 +1,8 @@
 """What the ops keep of static index maps: nothing while a graph is captured or
-of inference tensors."""
+of inference tensors, and nothing that outlives a change or goes with a copy."""
+import copy
+import pickle
+
 import pytest
 import torch
 
@@ -35,6 +38,28 @@ def test_kept(cpu_stream):
     assert get(d, m) is first and int(first[0]) == 10
     m[0] = 4
     assert int(get(d, m)[0]) == 14 and int(get(d, m.clone())[0]) == 14
+
+
+@pytest.mark.parametrize("copy_of", [copy.deepcopy, lambda x: pickle.loads(pickle.dumps(x))],
+                         ids=["copied", "saved"])
+def test_copies(cpu_stream, copy_of):
+    """A copy after a change: the copied map counts its own changes anew, and
+    may come to the count that the plan was made at."""
+    d, m, get = sums()
+    first = copy_of(m)._version
+    while m._version < first:
+        m[0] = 0
+    get(d, m)
+    m[0] = 4
+    d, m = copy_of((d, m))
+    assert int(get(d, m)[0]) == 14
+
+
+def test_other_storage(cpu_stream):
+    d, m, get = sums()
+    get(d, m)
+    m.data = torch.arange(7)
+    assert int(get(d, m)[0]) == 21
 
 
 def test_nothing_kept(cpu_stream, monkeypatch):
