@@ -248,14 +248,16 @@ class Derived:
     It holds the maps, so none can be replaced by another, and rebuilds after
     an in-place change (one that torch does not count, through .data or a raw
     pointer, is not seen).  A build is waited for, so that any stream may use
-    it.  A copy or a saved one holds nothing.
+    it, and what another one uses is freed only after it.  A copy or a saved
+    one holds nothing.
     get is None where nothing may be kept, and the caller works on the maps
     themselves: of inference tensors, whose changes are not counted, and while
     a graph is captured, which would only record a build and would hold the
     addresses of what a later change of the maps frees."""
 
     def __init__(self):
-        self._state = (None, None, None)  # maps, their versions and addresses, the value
+        # maps, their versions and addresses, the value, the stream that built it
+        self._state = (None, None, None, None)
 
     def __reduce__(self):
         return Derived, ()  # a copied map's versions start anew
@@ -264,12 +266,25 @@ class Derived:
         if any(m.is_inference() for m in maps) or torch.cuda.is_current_stream_capturing():
             return None
         key = tuple((m._version, m.data_ptr()) for m in maps)
-        held, seen, value = self._state
+        stream = stream_ptr(maps[0].device)
+        held, seen, value, built = self._state
         if held is None or any(a is not b for a, b in zip(held, maps)) or seen != key:
-            value = build(*maps)
+            value, built = build(*maps), stream
             torch.cuda.current_stream(maps[0].device).synchronize()
-            self._state = (maps, key, value)
+            self._state = (maps, key, value, built)
+        if stream != built:
+            for t in _tensors(value):
+                t.record_stream(torch.cuda.current_stream(maps[0].device))
         return value
+
+
+def _tensors(value):
+    """The tensors in a nest of tuples and dicts."""
+    if torch.is_tensor(value):
+        yield value
+    elif isinstance(value, (tuple, dict)):
+        for v in value.values() if isinstance(value, dict) else value:
+            yield from _tensors(v)
 
 
 class Workspace:

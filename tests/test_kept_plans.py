@@ -156,3 +156,34 @@ def test_few_positions(monkeypatch):
     for nodes in (3, 4, 5, 6):
         op(torch.rand(2 * nodes))
     assert taken == [None, None, "tiles", "tiles"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("least", [1, 1 << 40], ids=["tiles", "few"])
+def test_other_stream(gpu, monkeypatch, least):
+    """Modules that are dropped while another stream has yet to run their call:
+    what it reads is not given to a new tensor before it has."""
+    from dreamplace_amd import pin_pos, pin_weight_sum
+    print("case kept plans on another stream %d" % least, flush=True)
+    monkeypatch.setattr(pin_pos, "TILE_MIN_PINS", least)
+    monkeypatch.setattr(pin_weight_sum, "TILE_MIN_PINS", least)
+    pins, nphys, nets = 50000, 7000, 9000
+    p2n, order, start, p2e = netlist(gpu, pins, nphys, nets)
+    off, pos = torch.rand(pins, device=gpu), torch.rand(2 * nphys, device=gpu)
+    w = torch.rand(nets, device=gpu)
+    a = pin_pos.PinPos(off, off, p2n, order, start, nphys)
+    b = pin_weight_sum.PinWeightSum(order, start, p2e, nphys)
+    want = a(pos).clone(), b(w).clone()
+    kept = [t for d in (a._tiles, b._plan) for t in N._tensors(d._state[2])]
+    held = {t.data_ptr(): t.numel() * t.element_size() for t in kept}
+    assert (len(held) > 8) == (least == 1) and held
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(40000000)
+        got = a(pos), b(w)
+    del a, b, kept
+    new = [torch.zeros(n, dtype=torch.uint8, device=gpu) for n in held.values()]
+    assert not held.keys() & {t.data_ptr() for t in new}
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
