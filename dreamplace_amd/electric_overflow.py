@@ -228,6 +228,10 @@ class ElectricOverflow(nn.Module):
             self._filler_arg = N.host_doubles(self.uniform_filler)
         return self._filler_arg
 
+    def __getstate__(self):
+        # a ctypes array cannot be saved; it is formed again from uniform_filler
+        return dict(self.__dict__, _filler_arg=None)
+
     def run_code(self, num_filler_nodes=None):
         """The `algorithm` argument a density call with that many fillers
         (default all) runs with (scatter_algorithm)."""
