@@ -4,9 +4,10 @@ any other.
 
 ``SpectralPlan`` holds the twiddle tables or the cosine / sine matrices of an
 M x N grid for one arithmetic form ("fp64", "fp32" or "bf16x3"; the fast
-transforms of the last are FP32 throughout) and the scratch the transforms
-need; it wraps dp_dct2 / dp_idct2 / dp_idxst_idct / dp_idct_idxst and
-dp_poisson_solve of libdreamplace_amd.
+transforms of the last are FP32 throughout) and scratch for the transforms;
+it wraps dp_dct2 / dp_idct2 / dp_idxst_idct / dp_idct_idxst and
+dp_poisson_solve of libdreamplace_amd.  get_plan shares one plan per grid, form
+and device among all modules, threads and streams.
 """
 import torch
 
@@ -21,6 +22,17 @@ def data_dtype(precision):
     return torch.float64 if precision == "fp64" else torch.float32
 
 
+_is_capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing", None)
+
+
+def capturing():
+    """Whether a graph is being captured on the current stream."""
+    return _is_capturing is not None and _is_capturing()
+
+
+MAX_FREE = 4  # streams whose scratch a plan keeps (2048 x 2048 in FP32: 118 MB each)
+
+
 class SpectralPlan:
     def __init__(self, M, N_, precision, device):
         if precision not in N.PRECISIONS:
@@ -32,10 +44,33 @@ class SpectralPlan:
         self.dtype = data_dtype(precision)
         nbytes = N.query("dp_spectral_plan_bytes", self.M, self.N, self.code)
         self.plan = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
-        N.call("dp_spectral_plan_init", self.M, self.N, self.code, N.ptr(self.plan),
+        self._tables = N.ptr(self.plan)
+        N.call("dp_spectral_plan_init", self.M, self.N, self.code, self._tables,
                N.stream_ptr(self.device))
-        self.ws = torch.empty(N.query("dp_spectral_workspace_bytes", self.M, self.N, self.code),
-                              dtype=torch.uint8, device=self.device)
+        self.gpu = self.device.type == "cuda"
+        if self.gpu and not capturing():
+            # the tables, for whichever stream reads them first
+            torch.cuda.current_stream(self.device).synchronize()
+        self._ws_bytes = N.query("dp_spectral_workspace_bytes", self.M, self.N, self.code)
+        self._free = {}  # a stream's handle -> the scratch that its last call has left
+
+    def _take(self, stream):
+        """(scratch, its address, whether to keep it) for one call on `stream`, to
+        be given back (_give) once that is queued: what the last call on the same
+        stream has left, which the stream orders before this one; new memory where
+        another thread's call has it, or under capture, as a graph's replays keep
+        no order with the calls outside.  At most MAX_FREE streams' scratch is
+        kept."""
+        graph = self.gpu and capturing()
+        held = None if graph else self._free.pop(stream, None)
+        if held is None:
+            ws = torch.empty(self._ws_bytes, dtype=torch.uint8, device=self.device)
+            held = ws, ws.data_ptr(), not graph
+        return held
+
+    def _give(self, stream, held):
+        if held[2] and len(self._free) < MAX_FREE:
+            self._free[stream] = held
 
     def _check(self, x):
         N.require_gpu(x, name="SpectralPlan")
@@ -49,8 +84,10 @@ class SpectralPlan:
         x = self._check(x)
         if out is None:
             out = torch.empty(self.M, self.N, dtype=self.dtype, device=self.device)
-        N.call(name, self.code, N.ptr(self.plan), self.M, self.N, N.ptr(x), N.ptr(out),
-               N.ptr(self.ws), N.stream_ptr(self.device))
+        stream = N.stream_ptr(self.device)
+        held = self._take(stream)
+        N.call(name, self.code, self._tables, self.M, self.N, N.ptr(x), N.ptr(out), held[1], stream)
+        self._give(stream, held)
         return out
 
     def dct2(self, x, out=None):
@@ -76,9 +113,12 @@ class SpectralPlan:
             energy = torch.empty((), dtype=self.dtype, device=self.device) if compute_energy else None
         else:
             fx, fy, phi, energy = out
-        N.call("dp_poisson_solve", self.code, N.ptr(self.plan), self.M, self.N, N.ptr(d),
+        stream = N.stream_ptr(self.device)
+        held = self._take(stream)
+        N.call("dp_poisson_solve", self.code, self._tables, self.M, self.N, N.ptr(d),
                float(bin_size_x), float(bin_size_y), 1 if compute_potential else 0, N.ptr(fx),
-               N.ptr(fy), N.ptr(phi), N.ptr(energy), N.ptr(self.ws), N.stream_ptr(self.device))
+               N.ptr(fy), N.ptr(phi), N.ptr(energy), held[1], stream)
+        self._give(stream, held)
         return fx, fy, phi, energy
 
 
@@ -90,5 +130,7 @@ def get_plan(M, N_, precision, device):
     p = _plans.get(key)
     if p is None:
         p = SpectralPlan(M, N_, precision, device)
-        _plans[key] = p
+        # while a graph is captured the tables are only recorded: the graph's own
+        if not (p.gpu and capturing()):
+            _plans[key] = p
     return p
