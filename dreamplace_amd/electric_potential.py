@@ -61,7 +61,10 @@ class ElectricPotentialFunction(Function):
             op.density_map(pos)
         if op.backward == "adjoint":
             return op.energy_gradient(pos, ctx.potential_map, grad_pos), None
-        binned = ctx.workspace if op.binning_generation == ctx.binning else None
+        # under capture algorithm "global" gathers from the positions alone: another
+        # call on the op between two graphs' replays would have re-binned the cells
+        binned = (ctx.workspace if op.binning_generation == ctx.binning
+                  and not torch.cuda.is_current_stream_capturing() else None)
         grad = op.electric_force(pos, ctx.field_map_x, ctx.field_map_y, grad_pos, binned=binned)
         return grad, None
 
