@@ -233,8 +233,8 @@ constexpr int kReduceBlock = 256;
 constexpr int kReduceMaxBlocks = 16384;
 // Workgroups of the reductions that pair the x and y entries of a [2N]
 // per-node vector (the step-size norms, fused or not): thread t of the
-// grid-stride loop takes nodes t, t + grid, ...; every such reduction uses
-// this grid, so their sums are bit-identical.
+// grid-stride loop takes nodes t, t + grid, ...; every such reduction but that
+// of the node pass by tiles uses this grid, so their sums are bit-identical.
 inline int node_reduce_blocks(int64_t num_nodes) {
   int64_t b = (num_nodes + kReduceBlock - 1) / kReduceBlock;
   if (b < 1) b = 1;

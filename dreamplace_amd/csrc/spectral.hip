@@ -1508,12 +1508,14 @@ int dp_poisson_solve(int precision, const void* plan, int M, int N, const void* 
   }
   if (any_shape(precision, M, N)) {
     const int64_t t16 = ceil_div(M, 16) * ceil_div(N, 16);
+    // what the interface refuses: on grids of other sides, the energy beside the
+    // potential above 2048^2 (a partial sum per 16 x 16 tile once had no room)
     DP_REQUIRE(!energy || !compute_potential || mfma_shape(M, N) || t16 <= kReduceMaxBlocks,
                DP_ERR_UNSUPPORTED,
                "spectral: %d x %d grid needs the matrix-core path (sides multiple of %d) for the "
                "energy of the potential",
                M, N, BT);
-    // the energy's partials, one per 32 x 32 tile, have room up to 4096^2
+    // here the energy's partials, one per 32 x 32 tile, have room up to 4096^2
     if (!energy || ceil_div(M, 32) * ceil_div(N, 32) <= kReduceMaxBlocks)
       return (precision == DP_SPECTRAL_FP64 ? poisson_any<double> : poisson_any<float>)(
           plan, precision, M, N, density_map, bin_size_x, bin_size_y, compute_potential != 0,

@@ -18,7 +18,7 @@
 //
 // Net order is a static plan of the nets by degree (dp_wa_pack_slices).
 // k_wa_pins works on the other plan that the interface offers (dp_wa_pack_
-// nets): nets of at most 64 pins packed best-fit-decreasing by degree into
+// nets; for callers of the interface, and what the tests hold the slices to): nets of at most 64 pins packed best-fit-decreasing by degree into
 // groups of at most 64 pins, one wavefront per group and one lane per pin,
 // the per-net reductions through LDS.  Nets of more than 64 pins follow all
 // others in either order and are done by one wavefront each, in chunks.
@@ -956,9 +956,11 @@ __global__ void k_prep_slice_node(const int* __restrict__ flat_node2pin,
 // with farea >= 0 the fillers (n >= nphys: no pins, so pws[n] = 0, and one
 // area) take farea without loading either array (0 + c * farea is the same
 // value).
-// Thread t takes nodes t, t + grid, ...; with `partials` it also sums
-// (grad - g_prev)^2 over x and y in FP64, in k_step_norms's order (the
-// step-size denominator of step_nobb, NesterovAcceleratedGradientOptimizer.py:131).
+// With `partials` it also sums (grad - g_prev)^2 over x and y in FP64 (the
+// step-size denominator of step_nobb, NesterovAcceleratedGradientOptimizer.py:131):
+// k_node_grad, whose thread t takes nodes t, t + grid, ..., in k_step_norms's
+// order; k_node_grad_tiles by its tiles, an order of its own, as fixed, that
+// differs in the last FP64 bits.
 // fillers_done: the fillers' outputs are already final (the field gather
 // wrote them); they are only read back for the sum, or not visited at all.
 // The evaluation's last sums, by one workgroup more of the node pass: the

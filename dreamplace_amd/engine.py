@@ -366,7 +366,8 @@ def can_track_metrics(schedule, algorithm, num_bins_x, num_bins_y, padding, unif
 # 150 / 143, 3.1 million 192 / 178, 5.2 million 386 / 410, 9.6 million 433 / 467;
 # FP64: 106 / 73, 604 thousand 114 / 107, 3.1 million 266 / 281, 5.2 million
 # 651 / 637.  (A rule on pins and cells together, which takes two streams for 1.2
-# million pins with 11 million fillers, gave 280 there for 276.)
+# million pins with 11 million fillers, gave 280 there for 276.)  In FP64 neither
+# way is the quicker throughout from 0.6 to 5.2 million pins, by 2 to 6%.
 OVERLAP_MIN_PINS = 1 << 22
 
 # Pins from which the pins schedule permutes between node and net order in
@@ -487,8 +488,9 @@ class PlacementObjective:
         skips that store otherwise.  wirelength: "weighted_average" or
         "logsumexp" (PlaceObj.py:467-503); the log-sum-exp model runs on the
         "pins" and "unfused" schedules.  overlap (pins schedule): run the
-        wirelength forward on a second stream, concurrently with the density
-        chain it does not depend on; the node-gradient pass joins them.
+        wirelength forward of a netlist of OVERLAP_MIN_PINS pins or more on a
+        second stream, concurrently with the density chain it does not depend
+        on; the node-gradient pass joins them.
         track_metrics (pins schedule, tiled density, fillers of one size, no
         padding): every evaluation also leaves the placer's metrics at its
         positions in `metric_out` (FP64 {HPWL, overflow cost, max bin
@@ -577,10 +579,11 @@ class PlacementObjective:
         # a second stream (default priority) for the wirelength forward
         self.side = None
         self._side_stream = None
-        # where the wirelength pass forks off: before the scatter ("scatter",
-        # measured best: 0.729 ms at config 1 against 0.750 before the solve,
-        # 0.736 before the gather and 0.766-0.770 on one stream; 1.494 ms at
-        # config 4 against 1.524, 1.547 and 1.498-1.507), "solve" or "gather"
+        # where the wirelength pass forks off: before the scatter ("scatter"),
+        # "solve" or "gather".  With the kernels of then, 9.6 million pins and 13
+        # million cells: 0.729 ms, 0.750 before the solve, 0.736 before the
+        # gather, 0.766-0.770 on one stream; 53 million cells: 1.494, 1.524,
+        # 1.547, 1.498-1.507
         self.fork_at = "scatter"
         self.set_overlap(overlap)
         self.filler_ranges = None
@@ -646,7 +649,9 @@ class PlacementObjective:
 
     def set_overlap(self, on):
         """Run the pins schedule's wirelength forward on a second stream
-        (on=True) or on the caller's stream.  Either gives the same bits."""
+        (on=True; from OVERLAP_MIN_PINS pins on, below which that is slower and
+        it keeps to the caller's) or on the caller's stream.  Either gives the
+        same bits."""
         if on and self.schedule == "pins":
             if self._side_stream is None:
                 self._side_stream = torch.cuda.Stream(device=self.dd.device)
@@ -659,6 +664,7 @@ class PlacementObjective:
 
     @property
     def overlap(self):
+        """Whether the second stream is switched on (set_overlap)."""
         return self.side is not None
 
     def set_net_weights(self, w):

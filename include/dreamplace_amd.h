@@ -91,7 +91,7 @@ enum {
   DP_KERNEL_WA_FORWARD = 2,       /* k_wa_slices / k_wa_pins / k_nets */
   DP_KERNEL_WA_BACKWARD = 3,
   DP_KERNEL_PIN_POS_FORWARD = 4,
-  DP_KERNEL_PIN_POS_BACKWARD = 5, /* k_node_grad / k_wa_pin_pos_bwd / k_pin_pos_bwd / k_slot_sum */
+  DP_KERNEL_PIN_POS_BACKWARD = 5, /* k_node_grad / k_wa_pin_pos_bwd / k_pin_pos_bwd / k_tile_node_sum */
   DP_KERNEL_SPECTRAL_GEMM = 6,
   DP_KERNEL_DENSITY_CONVERT = 7,
   DP_KERNEL_DENSITY_BIN = 8,      /* k_bin_fill */
@@ -474,7 +474,13 @@ int dp_wa_backward_to_nodes(int dtype, const void* grad, const void* grad_interm
                             const uint8_t* pin_mask, const void* add, int64_t num_physical_nodes,
                             int64_t num_nodes, void* grad_pos_out, void* stream);
 
-/* Pin-parallel form of the fused wirelength chain (no reference counterpart:
+/* The group form, which ends with dp_lse_forward_pins and dp_wa_pins_slot_
+ * weights, dp_node_grad_from_pins, dp_node_grad_preconditioned and
+ * dp_hpwl_from_nets are kept for callers of this interface and as what the
+ * package's tests compare with; the package itself runs dp_wa_forward_slices or
+ * _tiles, dp_node_grad_objective and dp_step_metrics.
+ *
+ * Pin-parallel form of the fused wirelength chain (no reference counterpart:
  * the reference runs one thread per net, weighted_average_wirelength_cuda_
  * merged_kernel.cu:16-85).  Host routine, plain host memory, no GPU work:
  * packs the nets of 1..64 pins best-fit-decreasing by degree into groups of
@@ -629,8 +635,10 @@ int dp_wa_forward_slices(int dtype, int model, const void* pos, int64_t num_node
  * it (with node_tiles) or on derivatives in node order (node_tiles NULL), and,
  * with num_partials > 0, *wl_out = the sum of the partial sums that
  * dp_wa_forward_slices or _tiles left in the first bytes of its workspace for a
- * NULL wl_out, dp_wa_num_partials of them (num_net_tiles 0: slices), and with
- * obj_out *obj_out = wl + energy_weight * *energy.
+ * NULL wl_out, dp_wa_num_partials of them (num_net_tiles 0: slices, or tiles of
+ * nets above 64 pins alone), and with
+ * obj_out *obj_out = wl + energy_weight * *energy.  dg_norm2_out has the bits of
+ * dp_node_grad_preconditioned without node_tiles; with them its sum runs by tiles.
  * workspace: dp_wa_pins_workspace_bytes(num_pins, dtype).  At most 8192 tiles
  * of either order. */
 int dp_wa_tile_pins(int dtype);
