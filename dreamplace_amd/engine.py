@@ -543,6 +543,7 @@ class PlacementObjective:
             arithmetic=density_arith)
         self.density.compute_initial_density_map(dd.pos)
         self.plan = self.density.plan(dt, dev)
+        self.solve_ws = self.plan.scratch()
         n, P, E = dd.num_nodes, dd.num_pins, dd.num_nets
         M, Nb = self.density.num_bins_x, self.density.num_bins_y
         z = lambda *s, dtype=dt: torch.empty(*s, dtype=dtype, device=dev)
@@ -741,7 +742,8 @@ class PlacementObjective:
                           compute_potential=self.potential is not None
                           and (want_energy or self.density_backward == "adjoint"),
                           compute_energy=want_energy,
-                          out=(self.field_x, self.field_y, self.potential, self.energy))
+                          out=(self.field_x, self.field_y, self.potential, self.energy),
+                          ws=self.solve_ws)
 
     def _reduce_metrics(self, pos, s):
         """metric_out = {HPWL (design net weights, all nets of two or more

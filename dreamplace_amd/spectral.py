@@ -54,6 +54,10 @@ class SpectralPlan:
         self._ws_bytes = N.query("dp_spectral_workspace_bytes", self.M, self.N, self.code)
         self._free = {}  # a stream's handle -> the scratch that its last call has left
 
+    def scratch(self):
+        """Scratch for a caller whose calls are in order to keep (poisson's ws)."""
+        return torch.empty(self._ws_bytes, dtype=torch.uint8, device=self.device)
+
     def _take(self, stream):
         """(scratch, its address, whether to keep it) for one call on `stream`, to
         be given back (_give) once that is queued: what the last call on the same
@@ -64,7 +68,7 @@ class SpectralPlan:
         graph = self.gpu and capturing()
         held = None if graph else self._free.pop(stream, None)
         if held is None:
-            ws = torch.empty(self._ws_bytes, dtype=torch.uint8, device=self.device)
+            ws = self.scratch()
             held = ws, ws.data_ptr(), not graph
         return held
 
@@ -73,7 +77,8 @@ class SpectralPlan:
             self._free[stream] = held
 
     def _check(self, x):
-        N.require_gpu(x, name="SpectralPlan")
+        if not x.is_cuda:
+            N.require_gpu(x, name="SpectralPlan")
         if x.dtype != self.dtype:
             raise RuntimeError("SpectralPlan(%s) expects %s data, got %s" % (self.precision, self.dtype, x.dtype))
         if x.shape[-2:] != (self.M, self.N):
@@ -103,8 +108,9 @@ class SpectralPlan:
         return self.transform("dp_idct_idxst", x, out)
 
     def poisson(self, density_map, bin_size_x, bin_size_y, compute_potential=True,
-                compute_energy=True, out=None):
-        """(field_x, field_y, potential or None, energy 0-dim tensor or None)."""
+                compute_energy=True, out=None, ws=None):
+        """(field_x, field_y, potential or None, energy 0-dim tensor or None).
+        With out and ws (scratch()) a call allocates nothing."""
         d = self._check(density_map)
         if out is None:
             fx = torch.empty(self.M, self.N, dtype=self.dtype, device=self.device)
@@ -114,7 +120,7 @@ class SpectralPlan:
         else:
             fx, fy, phi, energy = out
         stream = N.stream_ptr(self.device)
-        held = self._take(stream)
+        held = self._take(stream) if ws is None else (ws, ws.data_ptr(), False)
         N.call("dp_poisson_solve", self.code, self._tables, self.M, self.N, N.ptr(d),
                float(bin_size_x), float(bin_size_y), 1 if compute_potential else 0, N.ptr(fx),
                N.ptr(fy), N.ptr(phi), N.ptr(energy), held[1], stream)
