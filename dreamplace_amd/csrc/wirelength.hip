@@ -216,8 +216,12 @@ struct NetSums {
     const T ax = lane_xor<O>(xmax), ay = lane_xor<O>(ymax);
     const T bx = lane_xor<O>(xmin), by = lane_xor<O>(ymin);
     if (!same) return;
-    extend(ax, ay);
-    extend(bx, by);
+    // each extreme with its own kind: pins that are not a number compare nowhere,
+    // and a lane of nothing but them still holds what it began with
+    xmax = ax > xmax ? ax : xmax;
+    ymax = ay > ymax ? ay : ymax;
+    xmin = bx < xmin ? bx : xmin;
+    ymin = by < ymin ? by : ymin;
   }
   template <int kModel, int O>
   __device__ __forceinline__ void join_sums(bool same) {

@@ -680,10 +680,16 @@ struct LaneNet {
     ymax = y > ymax ? y : ymax;
     ymin = y < ymin ? y : ymin;
   }
-  // combine with the lane `o` away, which holds other pins of the net
+  // combine with the lane `o` away, which holds other pins of the net; each
+  // extreme with its own kind, as a lane of nothing but pins that are not a number
+  // still holds what clear() left
   __device__ __forceinline__ void join_extremes(int o) {
-    extend(__shfl_xor(xmax, o), __shfl_xor(ymax, o));
-    extend(__shfl_xor(xmin, o), __shfl_xor(ymin, o));
+    const T ax = __shfl_xor(xmax, o), ay = __shfl_xor(ymax, o);
+    const T bx = __shfl_xor(xmin, o), by = __shfl_xor(ymin, o);
+    xmax = ax > xmax ? ax : xmax;
+    ymax = ay > ymax ? ay : ymax;
+    xmin = bx < xmin ? bx : xmin;
+    ymin = by < ymin ? by : ymin;
   }
   __device__ __forceinline__ void join_sums(int o) {
     if (kMode != kWaLse) {
