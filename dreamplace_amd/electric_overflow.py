@@ -56,9 +56,15 @@ class ElectricDensityMapFunction:
         if large_capacity is None:
             large_capacity = num_nodes
         cells = int(num_movable_nodes) + int(num_filler_nodes)
-        alg = algorithm_code(scatter_algorithm(algorithm, cells, nbx, nby), arithmetic)
-        nbytes = N.query("dp_density_map_workspace_bytes", nbx, nby, cells, int(large_capacity),
-                         alg, N.dtype_code(pos))
+        def sized(algorithm):
+            alg = algorithm_code(algorithm, arithmetic)
+            return alg, N.query("dp_density_map_workspace_bytes", nbx, nby, cells,
+                                int(large_capacity), alg, N.dtype_code(pos))
+
+        alg, nbytes = sized(scatter_algorithm(algorithm, cells, nbx, nby))
+        if workspace is not None and workspace.numel() < nbytes:
+            # a caller's own, sized for the algorithm that was asked for
+            alg, nbytes = sized(algorithm)
         if workspace is None or workspace.numel() < nbytes:
             workspace = N.workspace.get("density_map", nbytes, pos.device)
         init = initial_density_map
